@@ -243,6 +243,34 @@ __global__ __launch_bounds__(kRowsThreads) void import_kernel(Geo g, uint8_t *pa
   image_to_tile<D>(g, pages + region_base(g, page, kvh, kind), kind, p0 % g.page_tokens, TT, 0, n, img);
 }
 
+// The drop-in decode's scratch pages from contiguous K and V rows: page i
+// holds tokens page_tokens*i on, and workgroup (x, 0, 0) writes the block
+// table's entries, length and sequence id that the decode then reads.  (As
+// three copies from host memory, a stream synchronization and an import per
+// kind, a 1024-token call of 24 query and 4 kv heads took 58 us, with this
+// launch 30.)
+template <int D>
+__global__ __launch_bounds__(kRowsThreads) void flash_import_kernel(Geo g, uint8_t *pages, const uint8_t *k_rows,
+                                                                    const uint8_t *v_rows, int32_t len, int32_t *bt,
+                                                                    int32_t *seq_len, int32_t *seq_id) {
+  __shared__ __attribute__((aligned(16))) uint16_t img[RowsImage<D>::kBytes / 2];
+  constexpr int32_t RB = 2 * RowsImage<D>::kRowHalves;
+  const int32_t TT = tile_tokens(g.page_tokens), p0 = (int32_t)blockIdx.x * TT;
+  const int32_t kvh = (int32_t)blockIdx.y, kind = (int32_t)blockIdx.z;
+  const int32_t page = p0 / g.page_tokens, n = min(TT, len - p0);
+  if (kvh == 0 && kind == 0 && threadIdx.x == 0) {
+    if (p0 % g.page_tokens == 0) bt[page] = page;
+    if (blockIdx.x == 0) {
+      *seq_len = len;
+      *seq_id = 0;
+    }
+  }
+  if (n <= 0) return;
+  load_run(reinterpret_cast<uint8_t *>(img), (kind == 0 ? k_rows : v_rows) + ((int64_t)kvh * len + p0) * RB, n * RB);
+  __syncthreads();
+  image_to_tile<D>(g, pages + region_base(g, page, kvh, kind), kind, p0 % g.page_tokens, TT, 0, n, img);
+}
+
 __global__ __launch_bounds__(256) void f32_to_f16_kernel(const float *in, uint16_t *out, int64_t n,
                                                          int32_t rule) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -304,6 +332,19 @@ hipError_t launch_import(const Geo &g, uint8_t *pages, const int32_t *bt, int32_
     hipLaunchKernelGGL(import_kernel<256>, grid, dim3(kRowsThreads), 0, s, g, pages, bt, len, kind, rows, fault);
   else
     hipLaunchKernelGGL(import_kernel<128>, grid, dim3(kRowsThreads), 0, s, g, pages, bt, len, kind, rows, fault);
+  return hipGetLastError();
+}
+
+hipError_t launch_flash_import(const Geo &g, uint8_t *pages, const uint8_t *k_rows, const uint8_t *v_rows,
+                               int32_t len, int32_t *bt, int32_t *seq_len, int32_t *seq_id, hipStream_t s) {
+  const int64_t tiles = ((int64_t)len + tile_tokens(g.page_tokens) - 1) / tile_tokens(g.page_tokens);
+  const dim3 grid((unsigned)std::max<int64_t>(tiles, 1), (unsigned)g.kv_heads, 2);
+  if (g.head_dim == 256)
+    hipLaunchKernelGGL(flash_import_kernel<256>, grid, dim3(kRowsThreads), 0, s, g, pages, k_rows, v_rows, len, bt,
+                       seq_len, seq_id);
+  else
+    hipLaunchKernelGGL(flash_import_kernel<128>, grid, dim3(kRowsThreads), 0, s, g, pages, k_rows, v_rows, len, bt,
+                       seq_len, seq_id);
   return hipGetLastError();
 }
 

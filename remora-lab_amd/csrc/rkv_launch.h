@@ -31,6 +31,10 @@ hipError_t launch_gather(const Geo &g, const uint8_t *pages, const int32_t *bt, 
                          int32_t kind, uint8_t *rows, int32_t *fault, hipStream_t s);
 hipError_t launch_import(const Geo &g, uint8_t *pages, const int32_t *bt, int32_t len,
                          int32_t kind, const uint8_t *rows, int32_t *fault, hipStream_t s);
+// K and V rows of one sequence into pages in token order (64-token pages,
+// identity block table), and that table, the length and sequence id 0
+hipError_t launch_flash_import(const Geo &g, uint8_t *pages, const uint8_t *k_rows, const uint8_t *v_rows,
+                               int32_t len, int32_t *bt, int32_t *seq_len, int32_t *seq_id, hipStream_t s);
 hipError_t launch_f32_to_f16(const float *in, uint16_t *out, int64_t n, int32_t rule,
                              hipStream_t s);
 // block-table update: records [seq][W ids] x n_rows, then n_seqs lengths,

@@ -1332,31 +1332,14 @@ rkv_status rkv_flash_decode_q8(rkv_ctx *ctx, const rkv_flash_decode_params *p,
   if (rkv_status st = check_geometry(&s.g, op)) return st;
   uint8_t *base = static_cast<uint8_t *>(scratch);
   hipStream_t hs = as_stream(stream);
-  // identity block table, length and sequence id, written by a tiny upload
-  std::vector<int32_t> bt(s.n_pages);
-  for (int32_t i = 0; i < s.n_pages; ++i) bt[i] = i;
-  const int32_t meta[2] = {p->seq_len, 0};
-  hipError_t e;
-  if ((e = hipMemcpyAsync(base + s.bt_off, bt.data(), sizeof(int32_t) * s.n_pages,
-                          hipMemcpyHostToDevice, hs)) != hipSuccess)
-    return hip_fail(op, e);
-  if ((e = hipMemcpyAsync(base + s.len_off, &meta[0], sizeof(int32_t), hipMemcpyHostToDevice, hs)) !=
-      hipSuccess)
-    return hip_fail(op, e);
-  if ((e = hipMemcpyAsync(base + s.sid_off, &meta[1], sizeof(int32_t), hipMemcpyHostToDevice, hs)) !=
-      hipSuccess)
-    return hip_fail(op, e);
-  // the host copies above come from stack/vector memory: finish them first
-  if ((e = hipStreamSynchronize(hs)) != hipSuccess) return hip_fail(op, e);
+  // the rows into the scratch pages, with the identity block table, length
+  // and sequence id, in one launch
   const int32_t *dbt = reinterpret_cast<const int32_t *>(base + s.bt_off);
-  if (p->seq_len > 0) {
-    if (rkv_status st = rkv_import_q8(ctx, &s.g, base + s.pages_off, dbt, p->seq_len, RKV_K,
-                                      reinterpret_cast<const uint8_t *>(k_words), stream))
-      return st;
-    if (rkv_status st = rkv_import_q8(ctx, &s.g, base + s.pages_off, dbt, p->seq_len, RKV_V,
-                                      reinterpret_cast<const uint8_t *>(v_words), stream))
-      return st;
-  }
+  hipError_t e = rkv::launch_flash_import(
+      to_geo(&s.g), base + s.pages_off, reinterpret_cast<const uint8_t *>(k_words),
+      reinterpret_cast<const uint8_t *>(v_words), p->seq_len, reinterpret_cast<int32_t *>(base + s.bt_off),
+      reinterpret_cast<int32_t *>(base + s.len_off), reinterpret_cast<int32_t *>(base + s.sid_off), hs);
+  if (e != hipSuccess) return hip_fail(op, e);
   rkv_decode_args a = fd_args(p, s, base, query, out);
   a.workspace = base + s.ws_off;
   a.workspace_bytes = rkv_decode_workspace_bytes(&s.g, &a);

@@ -1,5 +1,7 @@
-"""Export and import at the edges of the tiles that their kernels move whole:
-part-filled tiles, odd row counts, pointers of any alignment.  Bit-exact."""
+"""Export, import, the drop-in decode's import and the R4KV spill at the edges
+of the tiles that their kernels move whole: part-filled tiles, odd row
+counts, output and input pointers of any alignment, several tiles per
+workgroup.  Bit-exact, except the drop-in's attention (f32 sums)."""
 import numpy as np
 import pytest
 
@@ -45,3 +47,36 @@ def test_gather_import_edges(rkv, rko, ctx, D, PT):
                 b = rko.paged_gather(lay, before, bt, full, k).reshape(Hkv, full, RB)
                 kept = slice(L, full) if k == kind else slice(0, full)
                 assert np.array_equal(a[:, kept], b[:, kept]), (L, shift, kind, k)
+
+
+@pytest.mark.parametrize("D", [128, 256])
+@pytest.mark.parametrize("L", [0, 1, 31, 64, 65, 300])
+def test_flash_decode_lengths(rkv, rko, ctx, D, L):
+    torch = _torch()
+    rng = np.random.default_rng(L + D)
+    Hq, Hkv = 6, 2
+    k, v = (rng.standard_normal((Hkv, L, D)).astype(np.float32) for _ in range(2))
+    q = (rng.standard_normal((Hq, D)) / np.sqrt(D)).astype(np.float32)
+    kr, vr = (np.frombuffer(b"".join(rko.q8_encode(x[h].reshape(-1)).tobytes() for h in range(Hkv)),
+                            np.uint8).copy() for x in (k, v))
+    p = rkv.FlashDecodeParams(Hq, Hkv, L, 1024, D)
+    scratch = torch.full((rkv.flash_decode_scratch_bytes(p),), 0xFF, dtype=torch.uint8, device="cuda")
+    out = torch.full((Hq, D), float("nan"), device="cuda")
+    qd = torch.from_numpy(q).cuda()
+    kd, vd = (torch.from_numpy(x).cuda() if L else None for x in (kr, vr))
+    for _ in range(2):  # the second call finds its own scratch of the first
+        rkv.flash_decode_q8(ctx, p, kd, vd, qd, out, scratch)
+    ctx.sync()
+    got = out.cpu().numpy()
+    if L == 0:
+        assert (got == 0).all()
+        return
+    blocks = [x.reshape(Hkv, L, D // 32, 34) for x in (kr, vr)]
+    kq, vq = ((b[..., 2:].view(np.int8).astype(np.float64) *
+               b[..., :2].copy().view(np.float16).astype(np.float64)).reshape(Hkv, L, D) for b in blocks)
+    for h in range(Hq):
+        s = kq[h // 3] @ q[h].astype(np.float64)
+        w = np.exp(s - s.max())
+        want = w @ vq[h // 3] / w.sum()
+        # f32 sums of up to 300 terms: well inside 1e-5 of the row's largest value
+        assert np.abs(got[h] - want).max() <= 1e-5 * np.abs(want).max()
