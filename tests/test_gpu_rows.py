@@ -80,3 +80,46 @@ def test_flash_decode_lengths(rkv, rko, ctx, D, L):
         want = w @ vq[h // 3] / w.sum()
         # f32 sums of up to 300 terms: well inside 1e-5 of the row's largest value
         assert np.abs(got[h] - want).max() <= 1e-5 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("D,PT,Hkv,layers,first,count", [
+    (128, 16, 4, 30, 7, 300),    # 3 tiles a workgroup, both edges part-filled
+    (128, 64, 1, 1, 33, 62),     # odd rows: runs at odd multiples of 8 bytes
+    (256, 64, 2, 48, 0, 640),    # whole tiles, 3 a workgroup
+    (256, 32, 2, 3, 31, 34),     # one row, a tile, one row
+    (256, 16, 3, 2, 5, 9),       # inside one tile
+    (256, 128, 8, 2, 0, 1),
+    (128, 32, 2, 2, 40, 0),      # no tokens: header and CRC of nothing
+])
+def test_spill_edges(rkv, ctx, D, PT, Hkv, layers, first, count):
+    torch = _torch()
+    n, RB = first + max(count, 1) + 3, rkv.row_bytes(D)
+    pages = (n + PT - 1) // PT
+    pool = rkv.Pool(ctx, layers, Hkv, D, PT, pages + 2, 1, pages, seed=3)
+    pool.alloc.reserve(0, n)
+    pool.sync_tables()
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(D + count)
+    pos = torch.arange(n, dtype=torch.int32, device="cuda")
+    for layer in range(layers):
+        k, v = (torch.randn((n, Hkv, D), generator=gen, device="cuda") for _ in range(2))
+        pool.append(layer, torch.zeros_like(pos), pos, k, v)
+    size = pool.r4kv_page_bytes(count, 0, layers - 1)
+    ident = rkv.R4kvHeader(prefix_digest=11, pos_start=first, epoch=1, generation=2)
+    staging = torch.full((size + 32,), 0xA5, dtype=torch.uint8, device="cuda")
+    for _ in range(2):  # the second spill finds the state the first left
+        pool.spill(0, first, count, 0, layers - 1, ident, staging, staging)
+    ctx.sync()
+    page = staging.cpu().numpy()
+    assert (page[size:] == 0xA5).all()
+    h, body = rkv.r4kv_unpack_host(page[:size])  # header, length and CRC
+    assert (h.token_start, h.token_count, h.layer_hi) == (first, count, layers - 1)
+    body = np.frombuffer(body, np.uint8).reshape(layers, 2, Hkv, count, RB)
+    rows = torch.empty(Hkv * n * RB, dtype=torch.uint8, device="cuda")
+    for layer in range(layers):
+        for kind in (0, 1):
+            pool.gather(layer, 0, kind, rows)
+            ctx.sync()
+            want = rows.cpu().numpy().reshape(Hkv, n, RB)[:, first:first + count]
+            assert np.array_equal(body[layer, kind], want), (layer, kind)
+    pool.close()
