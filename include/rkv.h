@@ -188,7 +188,7 @@ typedef struct rkv_decode_args {
   int32_t partition_tokens; /* split-K partition length: a multiple of max(32,
                                page_tokens), at most 64*page_tokens; 0 = chosen
                                per launch on the device from the batch's
-                               lengths (the smallest such length, >= 256,
+                               lengths (the smallest such length
                                whose partitions fill one round of resident
                                workgroups) */
   int32_t max_seq_len;      /* >= every seq_lens[seq_ids[b]]; sizes the grid */

@@ -2251,7 +2251,7 @@ __global__ __launch_bounds__(64 * NW, NW) void decode_kernel(DecodeLaunch p) {
 
 template <int D, int NT, int NS, int NW = 1>
 hipError_t launch_decode_t(const DecodeLaunch &d, hipStream_t s) {
-  dim3 grid((unsigned)d.n_wg, (unsigned)d.g.kv_heads);
+  dim3 grid((unsigned)d.n_grid, (unsigned)d.g.kv_heads);
   const bool small = d.g.page_tokens < kTile;
   if constexpr (NT == 2) {
     if (d.q_bf16 != 0) {

@@ -70,12 +70,13 @@ struct DecodeLaunch {
   // k*pt_unit (pt_unit = one 32-token tile), k in [pt_kmin, pt_kmax], whose
   // partition count over the batch is <= target_parts (else the longest);
   // a length whose partitions could start inside a page and span more than
-  // 64 pages rounds up to 64 pages.  Workgroup x of the grid (n_wg,
+  // 64 pages rounds up to 64 pages.  Workgroup x of the grid (n_grid,
   // kv_heads) takes the x-th partition of the batch in entry order.
   int32_t part_tokens;
   int32_t pt_unit, pt_kmin, pt_kmax, target_parts;
   int32_t max_len;  // >= every length of the batch
-  int32_t n_wg;     // upper bound of the batch's partition count
+  int32_t n_wg;     // upper bound of the batch's partition count, the flat layout's stride
+  int32_t n_grid;   // workgroups launched per kv head, <= n_wg
   int32_t n_parts;  // per-entry layout only: ceil(max_len / part_tokens)
   // direct output (ws_o == nullptr) ...
   void *out;

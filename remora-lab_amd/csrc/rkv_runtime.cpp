@@ -552,7 +552,7 @@ int32_t decode_stages() {
 
 // Partition plan of a decode launch (rkv::DecodeLaunch fields).  Explicit
 // partition_tokens fix the length; 0 leaves it to the kernel, which picks the
-// smallest whole number of 32-token tiles, at least 256 tokens and at most
+// smallest whole number of 32-token tiles, at least kmin of them and at most
 // 64 pages, whose partition count over the batch's actual lengths fills one
 // round of resident workgroups (target = resident slots / kv_heads).  Tile
 // granularity (not page) keeps the longest partition short: config 2's
@@ -561,17 +561,22 @@ struct Plan {
   int32_t pt = 0;  // explicit length, 0 = chosen on the device
   int32_t unit = 0, kmin = 0, kmax = 0, target = 0;
   int32_t max_len = 0;
-  int32_t n_wg = 0;     // grid.x: upper bound of the batch's partition count
+  int32_t n_wg = 0;     // upper bound of the batch's partition count: the partials' layout
+  int32_t n_grid = 0;   // grid.x: the same for this plan's shortest partition
   int32_t n_parts = 0;  // explicit: ceil(max_len / pt)
   bool direct = false;  // one partition covers every sequence: no partials
   int32_t stages = 2;   // LDS ring depth of the launch
 };
 
-Plan plan_of(const rkv_kv_geometry *g, const rkv_decode_args *a, int32_t stages) {
+constexpr int64_t kFewPartitions = 128;
+
+// whole: up to kWholeTiles tiles stay one partition (no partials).
+constexpr int32_t kWholeTiles = 8;
+
+Plan plan_of(const rkv_kv_geometry *g, const rkv_decode_args *a, int32_t stages, bool whole = false) {
   Plan pl;
   pl.stages = stages;
   pl.unit = 32;
-  pl.kmin = 256 / pl.unit;
   pl.kmax = 64 * g->page_tokens / pl.unit;
   pl.max_len = std::max<int32_t>(a->max_seq_len, 1);
   const int32_t rows = a->q_len * (a->q_heads / std::max(g->kv_heads, 1));
@@ -579,15 +584,37 @@ Plan plan_of(const rkv_kv_geometry *g, const rkv_decode_args *a, int32_t stages)
                         rkv::decode_wgs_per_cu(g->head_dim, rows, stages);
   pl.target = (int32_t)std::max<int64_t>(1, slots / g->kv_heads);
   const int64_t B = std::max<int32_t>(a->batch, 0);
+  // The shortest partition that the device may choose, in tiles.  A batch that
+  // does not fill the machine takes as many workgroups as it has shortest
+  // partitions, and each tile that a wave walks costs it 1.5 to 2 us (its
+  // loads land one tile at a time), while a longer list of partials costs the
+  // combine little.  Measured at 1, 2, 3, 4 and 8 tiles, us per call: 300
+  // tokens (D 128) 12.4, 13.8, 13.8, 14.7, 19.1; 1024 tokens of 4 kv heads
+  // 17.2, 19.6, 21.0, 22.6, 28.2; 32,768 tokens 22.1, 22.0, 20.7, 20.6, 24.4; 64
+  // sequences of 200 20.0, 17.6, 17.5, 18.1, 20.2; four drafts (32 rows) on 4
+  // x 1024 26.6, 24.0, 26.1, 21.8, 27.0.
+  const int32_t tiles = (pl.max_len + pl.unit - 1) / pl.unit;
+  pl.kmin = rows > 16 ? 4 : (B * tiles * g->kv_heads <= kFewPartitions ? 1 : 2);
   if (a->partition_tokens > 0) {
     pl.pt = a->partition_tokens;
     pl.n_parts = (pl.max_len + pl.pt - 1) / pl.pt;
     pl.n_wg = (int32_t)std::min<int64_t>(B * pl.n_parts, INT32_MAX);
+    pl.n_grid = pl.n_wg;
     pl.direct = pl.n_parts == 1;
   } else {
-    const int64_t pmax = (int64_t)pl.kmax * pl.unit;
-    pl.n_wg = (int32_t)std::min<int64_t>(
-        std::max<int64_t>(pl.target, B * ((pl.max_len + pmax - 1) / pmax)), INT32_MAX);
+    // A few tiles stay one partition where the combine launch costs more than
+    // the tiles that a split takes off the longest wave: about 4.5 us and 1.25
+    // per 1000 rows against 1.8 a tile (41 sequences of up to 161 tokens, 144
+    // rows each: 22.2 us in one partition, 32.8 split in two).
+    const int64_t out_rows = B * a->q_len * a->q_heads;
+    const int64_t in_one = whole ? kWholeTiles : std::min<int64_t>(kWholeTiles, pl.kmin + (3600 + out_rows) / 1440);
+    if (tiles <= in_one) pl.kmin = std::max(pl.kmin, tiles);
+    // The layout's bound follows batch and max_len alone, not kmin, so that a
+    // workspace that holds a call holds every smaller one.
+    const int64_t pmin = (int64_t)pl.kmin * pl.unit, pmax = (int64_t)pl.kmax * pl.unit;
+    const int64_t most = std::max<int64_t>(pl.target, B * ((pl.max_len + pmax - 1) / pmax));
+    pl.n_wg = (int32_t)std::min<int64_t>({most, std::max<int64_t>(B * tiles, 1), INT32_MAX});
+    pl.n_grid = (int32_t)std::min<int64_t>(pl.n_wg, std::max<int64_t>(B * ((pl.max_len + pmin - 1) / pmin), 1));
     pl.direct = pl.max_len <= pl.kmin * pl.unit;
   }
   return pl;
@@ -617,8 +644,14 @@ WsLayout ws_layout(const rkv_kv_geometry *g, const rkv_decode_args *a, const Pla
   const size_t prows = (size_t)g->kv_heads * pl.n_wg * batch_rows_per_kv(g, a);
   // partitions of one entry: ceil(max_len / shortest partition), and with a
   // device-chosen length no more than the target minus one per other entry
-  // (or the count at the longest length, where the search stops)
-  const int64_t shortest = pl.pt > 0 ? pl.pt : (int64_t)pl.kmin * pl.unit;
+  // (or the count at the longest length, where the search stops).  Shortest:
+  // what the device chooses when every entry is max_len long, up to the 8
+  // tiles below which only batches that do not fill the machine go (72
+  // sequences of about 2000 tokens, 9-tile partitions: 41.2 us with the one
+  // slice that this gives, 42.9 with two).
+  const int64_t even = ((int64_t)B * ((pl.max_len + 31) / 32) + pl.target - 1) / pl.target;
+  const int64_t shortest =
+      pl.pt > 0 ? pl.pt : std::max<int64_t>(pl.kmin, std::min<int64_t>(even, 8)) * pl.unit;
   int64_t n_entry = (pl.max_len + shortest - 1) / shortest;
   if (pl.pt == 0) {
     const int64_t longest = (int64_t)pl.kmax * pl.unit;
@@ -665,6 +698,7 @@ rkv::DecodeLaunch make_decode(rkv_ctx *ctx, const rkv_kv_geometry *g, const void
   d.target_parts = pl.target;
   d.max_len = pl.max_len;
   d.n_wg = pl.n_wg;
+  d.n_grid = pl.n_grid;
   d.n_parts = pl.n_parts;
   d.out = a->out;
   d.out_bf16 = a->out_dtype == RKV_BF16;
@@ -1098,7 +1132,11 @@ rkv_status decode_q8(rkv_ctx *ctx, const rkv_kv_geometry *g, const void *pages,
   if (rkv_status s = check_tables(pages, block_tables, bt_stride, n_seqs, op)) return s;
   if (!seq_lens) return fail(RKV_ERR_INVALID_ARG, op, "seq_lens is NULL");
   if (a->batch == 0) return RKV_OK;
-  const Plan pl = plan_of(g, a, stages);
+  Plan pl = plan_of(g, a, stages);
+  // short sequences need no workspace: without one they stay whole
+  if (pl.pt == 0 && !pl.direct && pl.max_len <= kWholeTiles * pl.unit &&
+      (!a->workspace || a->workspace_bytes < ws_bytes(g, a, pl)))
+    pl = plan_of(g, a, stages, true);
   rkv::DecodeLaunch d = make_decode(ctx, g, pages, block_tables, bt_stride, seq_lens, n_seqs, a, pl);
   hipStream_t hs = as_stream(stream);
   if (!pl.direct) {
@@ -1145,15 +1183,16 @@ rkv_status rkv_decode_q8_noalloc(rkv_ctx *ctx, const rkv_kv_geometry *g, const v
   if (rkv_status s = use_device(ctx, op)) return s;
   if (rkv_status s = check_decode(g, a, op)) return s;
   if (!ctx->scratch) return fail(RKV_ERR_DEVICE, op, "no static scratch on device %d", ctx->device);
-  const size_t need = ws_bytes(g, a, plan_of(g, a, decode_stages()));
+  // (short sequences stay whole, so their calls do not share the scratch)
+  const size_t need = ws_bytes(g, a, plan_of(g, a, decode_stages(), true));
   if (need > rkv::kDecodeScratchBytes)
     return fail(RKV_ERR_INVALID_ARG, op,
                 "the split-K partials need %zu bytes, more than the %zu-byte static scratch "
                 "(fewer entries, shorter max_seq_len or longer partitions fit; rkv_decode_q8 "
                 "takes a workspace of any size)", need, rkv::kDecodeScratchBytes);
   rkv_decode_args b = *a;
-  b.workspace = ctx->scratch;
-  b.workspace_bytes = rkv::kDecodeScratchBytes;
+  b.workspace = need > 0 ? ctx->scratch : nullptr;
+  b.workspace_bytes = need > 0 ? rkv::kDecodeScratchBytes : 0;
   return decode_q8(ctx, g, pages, block_tables, bt_stride, seq_lens, n_seqs, &b, stream,
                    decode_stages());
 }
