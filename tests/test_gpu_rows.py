@@ -123,3 +123,37 @@ def test_spill_edges(rkv, ctx, D, PT, Hkv, layers, first, count):
             want = rows.cpu().numpy().reshape(Hkv, n, RB)[:, first:first + count]
             assert np.array_equal(body[layer, kind], want), (layer, kind)
     pool.close()
+
+
+@pytest.mark.parametrize("D,PT,rows", [(128, 16, 8200), (256, 16, 8200), (256, 64, 8301), (256, 32, 300), (128, 64, 37)])
+def test_append_of_ragged_sequences(rkv, rko, ctx, D, PT, rows):
+    """Runs of rows that start and end at every slot modulo 4, in 32-row
+    workgroups (whole shifted quads, several sequences in one, a part-filled
+    last one, a last chunk of row blocks that is not full) and 8-row ones."""
+    torch = _torch()
+    rng = np.random.default_rng(rows + D + PT)
+    Hkv, sid, pos, ends = 8, [], [], []
+    while len(sid) < rows:
+        start = int(rng.integers(0, 70))
+        n = min(int(rng.choice([1, 3, 30, 61, 130, 515])), rows - len(sid))
+        sid += [len(ends)] * n
+        pos += range(start, start + n)
+        ends.append(start + n)
+    W = max(-(-e // PT) for e in ends)
+    need = sum(-(-e // PT) for e in ends)
+    bt = np.full((len(ends), W), -1, np.int32)
+    order, at = rng.permutation(need).astype(np.int32), 0
+    for s, e in enumerate(ends):
+        n = -(-e // PT)
+        bt[s, :n] = order[at:at + n]
+        at += n
+    sid, pos = np.array(sid, np.int32), np.array(pos, np.int32)
+    k, v = (rng.standard_normal((rows, Hkv, D)).astype(np.float32) for _ in range(2))
+    g = rkv.geometry(Hkv, D, PT, need)
+    before = rng.integers(0, 256, need * rkv.page_bytes(g), dtype=np.uint8)
+    pages = torch.from_numpy(before).cuda()
+    rkv.append_q8(ctx, g, pages, *(torch.from_numpy(x).cuda() for x in (bt, sid, pos, k, v)))
+    ctx.sync()
+    want = before.copy()
+    rko.paged_append(rko.layout(Hkv, D, PT, need), want, bt, sid, pos, k, v)
+    assert np.array_equal(pages.cpu().numpy(), want)
