@@ -187,14 +187,18 @@ typedef struct rkv_decode_args {
   int32_t out_dtype;        /* RKV_F32 | RKV_BF16 */
   int32_t partition_tokens; /* split-K partition length: a multiple of max(32,
                                page_tokens), at most 64*page_tokens; 0 = chosen
-                               per launch on the device from the batch's
-                               lengths (the smallest such length
-                               whose partitions fill one round of resident
-                               workgroups) */
+                               per launch: one partition while max_seq_len <=
+                               256; above that on the device, from the batch's
+                               lengths, the smallest whole number of 32-token
+                               tiles, at least 1, 2 or 4 by batch and rows and
+                               at most 64 pages, whose partitions fit one round
+                               of resident workgroups (the longest if none do) */
   int32_t max_seq_len;      /* >= every seq_lens[seq_ids[b]]; sizes the grid */
   void *workspace;          /* device scratch for the split-K partials, of
-                               rkv_decode_workspace_bytes (may be NULL when one
-                               partition covers every sequence) */
+                               rkv_decode_workspace_bytes.  Where that is 0 (one
+                               partition covers every sequence) it may be NULL
+                               and is not written; else calls that overlap need
+                               one each */
   size_t workspace_bytes;
   const rkv_append_args *append; /* optional (NULL = none): this step's K/V rows,
                                appended by the decode launch itself before it
@@ -208,7 +212,8 @@ typedef struct rkv_decode_args {
                                har-serve-vulkan-attn-smoke.rs:62-69, 149-161). */
   void *split_event;        /* optional hipEvent_t, recorded on the stream
                                between the decode kernel and the combine kernel
-                               (per-kernel timing); NULL = none */
+                               (per-kernel timing); NULL = none.  Not recorded by
+                               a call of workspace 0, which has no combine */
 } rkv_decode_args;
 
 /* Chunked prefill attention.  The reference's BatchStepModel::prefill_batch
@@ -276,15 +281,19 @@ rkv_status rkv_decode_q8(rkv_ctx *ctx, const rkv_kv_geometry *g, const void *pag
  * call on one device shares that array, and a call leaves its contents
  * behind (no call needs them cleared): calls that overlap on one device --
  * queued on different streams, or from several threads -- race and give
- * wrong results; calls queued on one stream are ordered. */
+ * wrong results; calls queued on one stream are ordered.  Only calls whose
+ * rkv_decode_workspace_bytes is 0 use none of it and may overlap. */
 #define RKV_DECODE_SCRATCH_BYTES ((size_t)64 << 20)
 rkv_status rkv_decode_q8_noalloc(rkv_ctx *ctx, const rkv_kv_geometry *g, const void *pages,
                                  const int32_t *block_tables, int32_t bt_stride,
                                  const int32_t *seq_lens, int32_t n_seqs,
                                  const rkv_decode_args *args, void *stream);
-/* Workspace bytes rkv_decode_q8 needs for these arguments (0 if none); it
- * depends on batch, q_len, q_heads, max_seq_len and partition_tokens, and
- * needs no initialisation. */
+/* Workspace bytes rkv_decode_q8 needs for these arguments; it depends on
+ * batch, q_len, q_heads, max_seq_len and partition_tokens, and needs no
+ * initialisation.  0 where one partition covers every sequence: with
+ * partition_tokens 0 up to a max_seq_len of 256, else up to one of
+ * partition_tokens.  With partition_tokens 0 it does not fall as batch or
+ * max_seq_len grows. */
 size_t rkv_decode_workspace_bytes(const rkv_kv_geometry *g, const rkv_decode_args *args);
 /* The explicit partition length of these arguments, or 0 when the device
  * chooses it per launch. */

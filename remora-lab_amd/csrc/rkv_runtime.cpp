@@ -570,10 +570,17 @@ struct Plan {
 
 constexpr int64_t kFewPartitions = 128;
 
-// whole: up to kWholeTiles tiles stay one partition (no partials).
+// Up to this many tiles (256 tokens) a batch stays one partition per entry.
+// Such a call neither needs nor writes a workspace, which is part of the
+// interface (rkv.h): calls that overlap may name the same one, and a result
+// has the same bits with and without one.  It costs short calls their split:
+// one sequence of 256 tokens (16 q / 2 kv heads, D 256) takes 20.5 us against
+// 14.6 in one-tile partitions, 64 sequences of 200 20.2 against 18.5.
 constexpr int32_t kWholeTiles = 8;
 
-Plan plan_of(const rkv_kv_geometry *g, const rkv_decode_args *a, int32_t stages, bool whole = false) {
+// own_scratch: the partials go to scratch that the call writes in any case
+// (the drop-in's), so the rule above does not hold it to one partition.
+Plan plan_of(const rkv_kv_geometry *g, const rkv_decode_args *a, int32_t stages, bool own_scratch = false) {
   Plan pl;
   pl.stages = stages;
   pl.unit = 32;
@@ -590,9 +597,8 @@ Plan plan_of(const rkv_kv_geometry *g, const rkv_decode_args *a, int32_t stages,
   // loads land one tile at a time), while a longer list of partials costs the
   // combine little.  Measured at 1, 2, 3, 4 and 8 tiles, us per call: 300
   // tokens (D 128) 12.4, 13.8, 13.8, 14.7, 19.1; 1024 tokens of 4 kv heads
-  // 17.2, 19.6, 21.0, 22.6, 28.2; 32,768 tokens 22.1, 22.0, 20.7, 20.6, 24.4; 64
-  // sequences of 200 20.0, 17.6, 17.5, 18.1, 20.2; four drafts (32 rows) on 4
-  // x 1024 26.6, 24.0, 26.1, 21.8, 27.0.
+  // 17.2, 19.6, 21.0, 22.6, 28.2; 32,768 tokens 22.1, 22.0, 20.7, 20.6, 24.4;
+  // four drafts (32 rows) on 4 x 1024 26.6, 24.0, 26.1, 21.8, 27.0.
   const int32_t tiles = (pl.max_len + pl.unit - 1) / pl.unit;
   pl.kmin = rows > 16 ? 4 : (B * tiles * g->kv_heads <= kFewPartitions ? 1 : 2);
   if (a->partition_tokens > 0) {
@@ -602,12 +608,12 @@ Plan plan_of(const rkv_kv_geometry *g, const rkv_decode_args *a, int32_t stages,
     pl.n_grid = pl.n_wg;
     pl.direct = pl.n_parts == 1;
   } else {
-    // A few tiles stay one partition where the combine launch costs more than
-    // the tiles that a split takes off the longest wave: about 4.5 us and 1.25
-    // per 1000 rows against 1.8 a tile (41 sequences of up to 161 tokens, 144
-    // rows each: 22.2 us in one partition, 32.8 split in two).
+    // With scratch of its own a call stays one partition only where the combine
+    // launch costs more than the tiles that a split takes off the longest wave:
+    // about 4.5 us and 1.25 per 1000 rows against 1.8 a tile.
     const int64_t out_rows = B * a->q_len * a->q_heads;
-    const int64_t in_one = whole ? kWholeTiles : std::min<int64_t>(kWholeTiles, pl.kmin + (3600 + out_rows) / 1440);
+    const int64_t in_one =
+        own_scratch ? std::min<int64_t>(kWholeTiles, pl.kmin + (3600 + out_rows) / 1440) : kWholeTiles;
     if (tiles <= in_one) pl.kmin = std::max(pl.kmin, tiles);
     // The layout's bound follows batch and max_len alone, not kmin, so that a
     // workspace that holds a call holds every smaller one.
@@ -1111,32 +1117,30 @@ int32_t rkv_decode_partition_tokens(const rkv_kv_geometry *g, const rkv_decode_a
   return a->partition_tokens > 0 ? a->partition_tokens : 0;
 }
 
-size_t rkv_decode_workspace_bytes(const rkv_kv_geometry *g, const rkv_decode_args *a) {
-  if (!g || !a || check_geometry(g, "rkv_decode_workspace_bytes") != RKV_OK) return 0;
-  if (a->q_heads < 1 || a->q_heads % g->kv_heads != 0 || a->q_len < 1) return 0;
-  // enough for either ring depth (a pool in host memory launches 3 stages)
-  return std::max(ws_bytes(g, a, plan_of(g, a, 2)), ws_bytes(g, a, plan_of(g, a, 3)));
-}
-
 }  // extern "C"
 
 namespace {
+size_t decode_ws_bytes(const rkv_kv_geometry *g, const rkv_decode_args *a, bool own_scratch) {
+  if (!g || !a || check_geometry(g, "rkv_decode_workspace_bytes") != RKV_OK) return 0;
+  if (a->q_heads < 1 || a->q_heads % g->kv_heads != 0 || a->q_len < 1) return 0;
+  // enough for either ring depth (a pool in host memory launches 3 stages)
+  return std::max(ws_bytes(g, a, plan_of(g, a, 2, own_scratch)), ws_bytes(g, a, plan_of(g, a, 3, own_scratch)));
+}
+
 // rkv_decode_q8 with an explicit LDS ring depth: 2 (the default, K codes in
 // registers) or 3 (K codes staged in LDS with V, two tiles in flight).
+// own_scratch: see plan_of.
 rkv_status decode_q8(rkv_ctx *ctx, const rkv_kv_geometry *g, const void *pages,
                      const int32_t *block_tables, int32_t bt_stride, const int32_t *seq_lens,
-                     int32_t n_seqs, const rkv_decode_args *a, void *stream, int32_t stages) {
+                     int32_t n_seqs, const rkv_decode_args *a, void *stream, int32_t stages,
+                     bool own_scratch = false) {
   const char *op = "rkv_decode_q8";
   if (rkv_status s = use_device(ctx, op)) return s;
   if (rkv_status s = check_decode(g, a, op)) return s;
   if (rkv_status s = check_tables(pages, block_tables, bt_stride, n_seqs, op)) return s;
   if (!seq_lens) return fail(RKV_ERR_INVALID_ARG, op, "seq_lens is NULL");
   if (a->batch == 0) return RKV_OK;
-  Plan pl = plan_of(g, a, stages);
-  // short sequences need no workspace: without one they stay whole
-  if (pl.pt == 0 && !pl.direct && pl.max_len <= kWholeTiles * pl.unit &&
-      (!a->workspace || a->workspace_bytes < ws_bytes(g, a, pl)))
-    pl = plan_of(g, a, stages, true);
+  const Plan pl = plan_of(g, a, stages, own_scratch);
   rkv::DecodeLaunch d = make_decode(ctx, g, pages, block_tables, bt_stride, seq_lens, n_seqs, a, pl);
   hipStream_t hs = as_stream(stream);
   if (!pl.direct) {
@@ -1167,6 +1171,10 @@ rkv_status decode_q8(rkv_ctx *ctx, const rkv_kv_geometry *g, const void *pages,
 
 extern "C" {
 
+size_t rkv_decode_workspace_bytes(const rkv_kv_geometry *g, const rkv_decode_args *a) {
+  return decode_ws_bytes(g, a, false);
+}
+
 rkv_status rkv_decode_q8(rkv_ctx *ctx, const rkv_kv_geometry *g, const void *pages,
                          const int32_t *block_tables, int32_t bt_stride,
                          const int32_t *seq_lens, int32_t n_seqs, const rkv_decode_args *a,
@@ -1183,16 +1191,15 @@ rkv_status rkv_decode_q8_noalloc(rkv_ctx *ctx, const rkv_kv_geometry *g, const v
   if (rkv_status s = use_device(ctx, op)) return s;
   if (rkv_status s = check_decode(g, a, op)) return s;
   if (!ctx->scratch) return fail(RKV_ERR_DEVICE, op, "no static scratch on device %d", ctx->device);
-  // (short sequences stay whole, so their calls do not share the scratch)
-  const size_t need = ws_bytes(g, a, plan_of(g, a, decode_stages(), true));
+  const size_t need = ws_bytes(g, a, plan_of(g, a, decode_stages()));
   if (need > rkv::kDecodeScratchBytes)
     return fail(RKV_ERR_INVALID_ARG, op,
                 "the split-K partials need %zu bytes, more than the %zu-byte static scratch "
                 "(fewer entries, shorter max_seq_len or longer partitions fit; rkv_decode_q8 "
                 "takes a workspace of any size)", need, rkv::kDecodeScratchBytes);
   rkv_decode_args b = *a;
-  b.workspace = need > 0 ? ctx->scratch : nullptr;
-  b.workspace_bytes = need > 0 ? rkv::kDecodeScratchBytes : 0;
+  b.workspace = ctx->scratch;
+  b.workspace_bytes = rkv::kDecodeScratchBytes;
   return decode_q8(ctx, g, pages, block_tables, bt_stride, seq_lens, n_seqs, &b, stream,
                    decode_stages());
 }
@@ -1342,8 +1349,7 @@ rkv_decode_args fd_args(const rkv_flash_decode_params *p, const FdScratch &s, ui
   a.out = out;
   a.out_dtype = RKV_F32;
   a.max_seq_len = p->seq_len;
-  // one partition covers the sequence when it fits 64 pages; else split
-  a.partition_tokens = 0;
+  a.partition_tokens = 0;  // chosen per call: see plan_of
   return a;
 }
 }  // namespace
@@ -1352,7 +1358,7 @@ size_t rkv_flash_decode_scratch_bytes(const rkv_flash_decode_params *p) {
   if (!p || p->seq_len < 0 || p->kv_heads < 1) return 0;
   FdScratch s = fd_scratch(p);
   rkv_decode_args a = fd_args(p, s, nullptr, nullptr, nullptr);
-  return s.total + rkv_decode_workspace_bytes(&s.g, &a);
+  return s.total + decode_ws_bytes(&s.g, &a, true);
 }
 
 rkv_status rkv_flash_decode_q8(rkv_ctx *ctx, const rkv_flash_decode_params *p,
@@ -1381,9 +1387,9 @@ rkv_status rkv_flash_decode_q8(rkv_ctx *ctx, const rkv_flash_decode_params *p,
   if (e != hipSuccess) return hip_fail(op, e);
   rkv_decode_args a = fd_args(p, s, base, query, out);
   a.workspace = base + s.ws_off;
-  a.workspace_bytes = rkv_decode_workspace_bytes(&s.g, &a);
-  return rkv_decode_q8(ctx, &s.g, base + s.pages_off, dbt, s.n_pages,
-                       reinterpret_cast<const int32_t *>(base + s.len_off), 1, &a, stream);
+  a.workspace_bytes = decode_ws_bytes(&s.g, &a, true);
+  return decode_q8(ctx, &s.g, base + s.pages_off, dbt, s.n_pages,
+                   reinterpret_cast<const int32_t *>(base + s.len_off), 1, &a, stream, decode_stages(), true);
 }
 
 }  // extern "C"

@@ -207,3 +207,20 @@ def test_decode_workspace_monotone(rkv, kv_heads, q_heads, D, PT, max_decode, ma
         w_top = _ws(rkv, g, B, max_len, q_heads)
         assert w_top >= prev_b, ("not monotone in batch", B)
         prev_b = w_top
+
+
+@pytest.mark.parametrize("kv_heads,q_heads,D,PT", [(2, 16, 256, 32), (1, 1, 128, 16), (8, 32, 128, 64), (4, 24, 256, 128)])
+def test_short_calls_ask_for_no_workspace(rkv, kv_heads, q_heads, D, PT):
+    """Up to 256 tokens a device-chosen plan is one partition: no workspace, at
+    any batch and q_len, so that one sized for a loop's largest call holds the
+    short ones too.  Explicit partitions need theirs at any length."""
+    g = rkv.geometry(kv_heads, D, PT, 1 << 20)
+    for q_len in (1, 2, 4):
+        prev = {}
+        for L in (0, 1, 31, 32, 33, 64, 97, 128, 129, 160, 200, 255, 256, 257, 288, 289, 600, 4096, 4097):
+            sizes = [_ws(rkv, g, B, L, q_heads, q_len) for B in (1, 2, 3, 8, 41, 64, 512)]
+            assert (max(sizes) == 0) == (L <= 256), (q_len, L, sizes)
+            assert sizes == sorted(sizes), (q_len, L, sizes)
+            assert not prev or all(x <= y for x, y in zip(prev[q_len], sizes)), (q_len, L)
+            prev[q_len] = sizes
+        assert _ws(rkv, g, 1, 256, q_heads, q_len, pt=max(32, PT)) > 0
