@@ -165,9 +165,9 @@ hipError_t launch_crc32c(const uint8_t *data, int64_t n, uint32_t *out, hipStrea
 // R4KV page body <-> pool: rows of tokens [t0, t0+count) of one sequence
 // (block-table row `bt`), layers [layer_lo, layer_lo+n_layers) of page
 // arrays layer_stride bytes apart.  Pack writes header, body and payload
-// CRC to page_out, through the two words of `state` (zero before the first
-// launch; each launch leaves them zero, and launches that share them run one
-// after the other); unpack writes a verified body back.
+// CRC to page_out, through the two words of `state`, which it clears first
+// (calls that share them run one after the other); unpack writes a verified
+// body back.
 struct R4kvLaunch {
   Geo g;
   int64_t layer_stride;

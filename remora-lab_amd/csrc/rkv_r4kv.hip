@@ -194,7 +194,16 @@ __device__ __forceinline__ uint32_t wave_shift(uint32_t c, uint64_t d, int lane)
   return c;
 }
 
-// Spill: the header, the body and the body's CRC32C in one launch.  Each
+// Opens a spill: the header, and the state that its workgroups share cleared,
+// so that no launch relies on what another left there (captured spills that
+// are replayed on two streams at once spoil each other's CRC; later ones must
+// not inherit it).  1.7 us.
+__global__ void spill_begin_kernel(Header96 h96, uint8_t *page_out, uint32_t *state) {
+  if (threadIdx.x < 24) reinterpret_cast<uint32_t *>(page_out)[threadIdx.x] = h96.w[threadIdx.x];
+  if (threadIdx.x < 2) state[threadIdx.x] = 0u;
+}
+
+// Spill: the body and its CRC32C in one launch.  Each
 // tile's rows leave for the body from the LDS image, and the CRC is taken
 // from the same image, so the body is not read back (the CRC as a second
 // pass over a 214 MB page took 115 us after a 128 us pack, and three one-word
@@ -209,10 +218,10 @@ __device__ __forceinline__ uint32_t wave_shift(uint32_t c, uint64_t d, int lane)
 // words: it is checksummed with slicing tables, moved to the body's end
 // (128*L bytes less than the part's distance from it; x has order 2^31 - 1,
 // which makes a negative shift a positive one) and xor-ed into state[0].  The
-// workgroup that counts the last adds the finishing term, stores the page's
-// trailing word and clears the state for the next launch.
+// workgroup that counts the last adds the finishing term and stores the page's
+// trailing word.
 template <int D, int TT>
-__global__ __launch_bounds__(kRowsThreads) void pack_kernel(BodyMap m, Header96 h96, const uint8_t *pages,
+__global__ __launch_bounds__(kRowsThreads) void pack_kernel(BodyMap m, const uint8_t *pages,
                                                             const int32_t *bt, uint8_t *page_out, int64_t body_len,
                                                             uint32_t finish, uint32_t *state, int32_t *fault) {
   constexpr int kLanes = TT * D / 64;
@@ -225,8 +234,6 @@ __global__ __launch_bounds__(kRowsThreads) void pack_kernel(BodyMap m, Header96 
   const int tid = threadIdx.x;
   for (int i = tid; i < 4 * 256; i += kRowsThreads) ts[i >> 8][i & 255] = c_slice16.t[i >> 8][i & 255];
   uint8_t *body = page_out + 96;
-  const bool first_wg = blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0;
-  if (first_wg && tid < 24) reinterpret_cast<uint32_t *>(page_out)[tid] = h96.w[tid];
   int32_t j0 = (int32_t)blockIdx.x * m.per, j1 = min(j0 + m.per, m.n_main);
   if (j0 >= m.n_main) {  // the last workgroup of a stream: its partly covered last tile
     j0 = m.n_main;
@@ -338,10 +345,8 @@ __global__ __launch_bounds__(kRowsThreads) void pack_kernel(BodyMap m, Header96 
   const uint32_t before = atomicXor(&state[0], acc);
   asm volatile("" : "+v"(one) : "v"(before));
   const uint32_t wgs = gridDim.x * gridDim.y * gridDim.z;
-  if (atomicAdd(&state[1], one) == wgs - 1) {
-    *reinterpret_cast<uint32_t *>(body + body_len) = atomicExch(&state[0], 0u) ^ finish;
-    atomicExch(&state[1], 0u);
-  }
+  if (atomicAdd(&state[1], one) == wgs - 1)
+    *reinterpret_cast<uint32_t *>(body + body_len) = atomicXor(&state[0], 0u) ^ finish;
 }
 
 template <int D>
@@ -406,8 +411,9 @@ hipError_t launch_r4kv_pack(const R4kvLaunch &r, const uint8_t *pages, const int
   const int32_t chunks = std::max<int32_t>(1, (m.n_main + m.per - 1) / m.per) + (lone ? 1 : 0);
   const dim3 grid((unsigned)chunks, (unsigned)(2 * r.g.kv_heads), (unsigned)m.n_layers);
   const uint32_t finish = crc::finish_term((uint64_t)body_len);
+  hipLaunchKernelGGL(spill_begin_kernel, dim3(1), dim3(64), 0, s, h, page_out, state);
   auto go = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, grid, dim3(kRowsThreads), 0, s, m, h, pages, bt, page_out, body_len, finish, state,
+    hipLaunchKernelGGL(kernel, grid, dim3(kRowsThreads), 0, s, m, pages, bt, page_out, body_len, finish, state,
                        fault);
   };
   if (r.g.head_dim == 256) {

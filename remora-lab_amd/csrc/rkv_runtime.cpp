@@ -1565,7 +1565,6 @@ rkv_status rkv_pool_create(rkv_ctx *ctx, const rkv_pool_desc *desc, rkv_pool **o
       (e = hipMemset(p->scatter_count, 0, sizeof(unsigned long long))) != hipSuccess ||
       (e = hipEventCreateWithFlags(&p->handoff, hipEventDisableTiming)) != hipSuccess ||
       (e = hipMalloc(&p->d_crc, 256)) != hipSuccess ||
-      (e = hipMemset(p->d_crc, 0, 256)) != hipSuccess ||
       (e = hipHostMalloc(&p->h_crc, 256, hipHostMallocDefault)) != hipSuccess) {
     rkv_status s = fail(RKV_ERR_DEVICE, op, "allocating %zu page bytes and tables: %s",
                         p->layer_bytes * desc->layers, hipGetErrorString(e));

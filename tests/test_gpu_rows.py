@@ -125,6 +125,60 @@ def test_spill_edges(rkv, ctx, D, PT, Hkv, layers, first, count):
     pool.close()
 
 
+def test_spill_after_overlapping_replays(rkv, ctx):
+    """Captured spills of one pool, replayed one at a time, give whole pages.
+    Replayed on two streams at once they may spoil each other's CRC word (a
+    restore refuses such a page), but no later spill's."""
+    torch = _torch()
+    layers, Hkv, D, PT, n = 8, 2, 256, 64, 2000
+    W = -(-n // PT)
+    pool = rkv.Pool(ctx, layers, Hkv, D, PT, W, 1, W, seed=9)
+    pool.alloc.reserve(0, n)
+    pool.sync_tables()
+    pos = torch.arange(n, dtype=torch.int32, device="cuda")
+    for layer in range(layers):
+        k, v = (torch.randn((n, Hkv, D), device="cuda") for _ in range(2))
+        pool.append(layer, torch.zeros_like(pos), pos, k, v)
+    ident = rkv.R4kvHeader(prefix_digest=3, pos_start=0, epoch=1, generation=1)
+    size = [pool.r4kv_page_bytes(c, 0, layers - 1) for c in (n, n - 33)]
+    staging = [torch.zeros(x, dtype=torch.uint8, device="cuda") for x in size]
+    streams = [torch.cuda.Stream() for _ in range(2)]
+
+    def spill(i, stream=None):
+        pool.spill(0, 0, n - 33 * i, 0, layers - 1, ident, staging[i], staging[i], stream=stream)
+
+    def whole(i):
+        rkv.r4kv_unpack_host(staging[i].cpu().numpy())  # raises unless header and CRC hold
+
+    graphs = []
+    for i, s in enumerate(streams):
+        spill(i, s)
+        torch.cuda.synchronize()
+        whole(i)
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=s):
+            spill(i, s)
+        graphs.append(g)
+    for i in (0, 1, 0):
+        staging[i].zero_()
+        torch.cuda.synchronize()
+        graphs[i].replay()
+        torch.cuda.synchronize()
+        whole(i)
+    for _ in range(20):
+        for g, s in zip(graphs, streams):
+            with torch.cuda.stream(s):
+                g.replay()
+    torch.cuda.synchronize()
+    for i in (0, 1):
+        staging[i].zero_()
+        spill(i)
+        ctx.sync()
+        whole(i)
+    del graphs
+    pool.close()
+
+
 @pytest.mark.parametrize("D,PT,rows", [(128, 16, 8200), (256, 16, 8200), (256, 64, 8301), (256, 32, 300), (128, 64, 37)])
 def test_append_of_ragged_sequences(rkv, rko, ctx, D, PT, rows):
     """Runs of rows that start and end at every slot modulo 4, in 32-row
