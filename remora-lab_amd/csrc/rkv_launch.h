@@ -165,9 +165,8 @@ hipError_t launch_crc32c(const uint8_t *data, int64_t n, uint32_t *out, hipStrea
 // R4KV page body <-> pool: rows of tokens [t0, t0+count) of one sequence
 // (block-table row `bt`), layers [layer_lo, layer_lo+n_layers) of page
 // arrays layer_stride bytes apart.  Pack writes header, body and payload
-// CRC to page_out, through the two words of `state`, which it clears first
-// (calls that share them run one after the other); unpack writes a verified
-// body back.
+// CRC (through crc_word, which it clears first; calls that share it run one
+// after the other) to page_out; unpack writes a verified body back.
 struct R4kvLaunch {
   Geo g;
   int64_t layer_stride;
@@ -176,7 +175,7 @@ struct R4kvLaunch {
   uint8_t header[96];
 };
 hipError_t launch_r4kv_pack(const R4kvLaunch &r, const uint8_t *pages, const int32_t *bt,
-                            uint8_t *page_out, uint32_t *state, int32_t *fault, hipStream_t s);
+                            uint8_t *page_out, uint32_t *crc_word, int32_t *fault, hipStream_t s);
 hipError_t launch_r4kv_unpack(const R4kvLaunch &r, uint8_t *pages, const int32_t *bt,
                               const uint8_t *body, int32_t *fault, hipStream_t s);
 // HBM streaming-read ceiling (rkv_stream.hip): mode 0 vector loads with the

@@ -194,13 +194,21 @@ __device__ __forceinline__ uint32_t wave_shift(uint32_t c, uint64_t d, int lane)
   return c;
 }
 
-// Opens a spill: the header, and the state that its workgroups share cleared,
-// so that no launch relies on what another left there (captured spills that
-// are replayed on two streams at once spoil each other's CRC; later ones must
-// not inherit it).  1.7 us.
-__global__ void spill_begin_kernel(Header96 h96, uint8_t *page_out, uint32_t *state) {
+// The launches before and behind pack_kernel: the header and a cleared CRC
+// word, so that no spill relies on what another left there (captured spills
+// that are replayed on two streams at once spoil each other's CRC; later ones
+// must not inherit it), then the page's trailing word.  The stream orders the
+// three, so that pack_kernel's xors need no order among themselves.  214 MB:
+// 125.6 us with the header and the trailing word in pack_kernel (its last
+// workgroup by a count), 127.3 with the first launch, 128.2 with both; a count
+// with acquire-release order, which writes an XCD's L2 back once per
+// workgroup, 197.6.
+__global__ void spill_begin_kernel(Header96 h96, uint8_t *page_out, uint32_t *crc_word) {
   if (threadIdx.x < 24) reinterpret_cast<uint32_t *>(page_out)[threadIdx.x] = h96.w[threadIdx.x];
-  if (threadIdx.x < 2) state[threadIdx.x] = 0u;
+  if (threadIdx.x == 0) *crc_word = 0u;
+}
+__global__ void spill_end_kernel(const uint32_t *crc_word, uint32_t finish, uint8_t *to) {
+  *reinterpret_cast<uint32_t *>(to) = *crc_word ^ finish;
 }
 
 // Spill: the body and its CRC32C in one launch.  Each
@@ -217,13 +225,11 @@ __global__ void spill_begin_kernel(Header96 h96, uint8_t *page_out, uint32_t *st
 // message of 32*L words, congruent to the part followed by as many zero
 // words: it is checksummed with slicing tables, moved to the body's end
 // (128*L bytes less than the part's distance from it; x has order 2^31 - 1,
-// which makes a negative shift a positive one) and xor-ed into state[0].  The
-// workgroup that counts the last adds the finishing term and stores the page's
-// trailing word.
+// which makes a negative shift a positive one) and xor-ed into the CRC word.
 template <int D, int TT>
 __global__ __launch_bounds__(kRowsThreads) void pack_kernel(BodyMap m, const uint8_t *pages,
                                                             const int32_t *bt, uint8_t *page_out, int64_t body_len,
-                                                            uint32_t finish, uint32_t *state, int32_t *fault) {
+                                                            uint32_t *crc_word, int32_t *fault) {
   constexpr int kLanes = TT * D / 64;
   constexpr int RB = 2 * RowsImage<D>::kRowHalves;
   static_assert(kLanes * kTileWords * 4 == TT * RB && kLanes <= kRowsThreads, "17 words a lane");
@@ -338,15 +344,7 @@ __global__ __launch_bounds__(kRowsThreads) void pack_kernel(BodyMap m, const uin
   int64_t d = body_len - end - 128 * kLanes;
   if (d < 0) d += 0x7fffffff;
   acc = wave_shift((uint32_t)__builtin_amdgcn_readfirstlane((int)acc), j1 > j0 ? (uint64_t)d : 0, lane);
-  if (tid != 0) return;
-  // the count follows the xor by its returned value: a device fence would
-  // write the XCD's whole L2 back, once per workgroup
-  uint32_t one = 1;
-  const uint32_t before = atomicXor(&state[0], acc);
-  asm volatile("" : "+v"(one) : "v"(before));
-  const uint32_t wgs = gridDim.x * gridDim.y * gridDim.z;
-  if (atomicAdd(&state[1], one) == wgs - 1)
-    *reinterpret_cast<uint32_t *>(body + body_len) = atomicXor(&state[0], 0u) ^ finish;
+  if (tid == 0) atomicXor(crc_word, acc);
 }
 
 template <int D>
@@ -392,7 +390,7 @@ hipError_t launch_crc32c(const uint8_t *data, int64_t n, uint32_t *out, hipStrea
 }
 
 hipError_t launch_r4kv_pack(const R4kvLaunch &r, const uint8_t *pages, const int32_t *bt,
-                            uint8_t *page_out, uint32_t *state, int32_t *fault, hipStream_t s) {
+                            uint8_t *page_out, uint32_t *crc_word, int32_t *fault, hipStream_t s) {
   BodyMap m = body_map(r);
   Header96 h;
   for (int i = 0; i < 24; ++i)
@@ -411,10 +409,9 @@ hipError_t launch_r4kv_pack(const R4kvLaunch &r, const uint8_t *pages, const int
   const int32_t chunks = std::max<int32_t>(1, (m.n_main + m.per - 1) / m.per) + (lone ? 1 : 0);
   const dim3 grid((unsigned)chunks, (unsigned)(2 * r.g.kv_heads), (unsigned)m.n_layers);
   const uint32_t finish = crc::finish_term((uint64_t)body_len);
-  hipLaunchKernelGGL(spill_begin_kernel, dim3(1), dim3(64), 0, s, h, page_out, state);
+  hipLaunchKernelGGL(spill_begin_kernel, dim3(1), dim3(64), 0, s, h, page_out, crc_word);
   auto go = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, grid, dim3(kRowsThreads), 0, s, m, pages, bt, page_out, body_len, finish, state,
-                       fault);
+    hipLaunchKernelGGL(kernel, grid, dim3(kRowsThreads), 0, s, m, pages, bt, page_out, body_len, crc_word, fault);
   };
   if (r.g.head_dim == 256) {
     if (TT == 32) go(pack_kernel<256, 32>);
@@ -423,6 +420,7 @@ hipError_t launch_r4kv_pack(const R4kvLaunch &r, const uint8_t *pages, const int
     if (TT == 32) go(pack_kernel<128, 32>);
     else go(pack_kernel<128, 16>);
   }
+  hipLaunchKernelGGL(spill_end_kernel, dim3(1), dim3(1), 0, s, crc_word, finish, page_out + 96 + body_len);
   return hipGetLastError();
 }
 

@@ -1398,7 +1398,7 @@ rkv_status rkv_flash_decode_q8(rkv_ctx *ctx, const rkv_flash_decode_params *p,
 // pool
 // ---------------------------------------------------------------------------
 namespace {
-constexpr int kSpillState = 32;  // on a line of its own
+constexpr int kSpillCrc = 32;  // word of rkv_pool::d_crc, on a line of its own
 }
 struct rkv_pool {
   rkv_ctx *ctx = nullptr;
@@ -1430,7 +1430,7 @@ struct rkv_pool {
   unsigned long long scatter_blocks = 0;
   uint32_t n_syncs = 0;
   // R4KV page CRC: device result word and its pinned host copy
-  uint32_t *d_crc = nullptr;  // word 0: a restore's CRC; kSpillState on: the spill's two words
+  uint32_t *d_crc = nullptr;  // word 0: a restore's CRC; kSpillCrc: a spill's
   uint32_t *h_crc = nullptr;
   // the stream of the pool's last call (see order_after_last)
   hipStream_t last_stream = nullptr;
@@ -2038,7 +2038,7 @@ rkv_status rkv_pool_spill(rkv_pool *p, int32_t seq, int32_t token_start, int32_t
   hipStream_t hs = as_stream(stream);
   if (rkv_status s = order_after_last(p, hs, op)) return s;
   hipError_t e = rkv::launch_r4kv_pack(r, p->pages, p->d_tables + (size_t)seq * p->d.max_pages_per_seq,
-                                       static_cast<uint8_t *>(staging), p->d_crc + kSpillState,
+                                       static_cast<uint8_t *>(staging), p->d_crc + kSpillCrc,
                                        p->ctx->d_fault, hs);
   if (e != hipSuccess) return hip_fail(op, e);
   if (dst != staging && (e = hipMemcpyAsync(dst, staging, need, hipMemcpyDefault, hs)) != hipSuccess)
