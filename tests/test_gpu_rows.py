@@ -50,7 +50,7 @@ def test_gather_import_edges(rkv, rko, ctx, D, PT):
 
 
 @pytest.mark.parametrize("D", [128, 256])
-@pytest.mark.parametrize("L", [0, 1, 31, 64, 65, 300])
+@pytest.mark.parametrize("L", [0, 1, 31, 64, 65, 96, 97, 200, 256, 300])
 def test_flash_decode_lengths(rkv, rko, ctx, D, L):
     torch = _torch()
     rng = np.random.default_rng(L + D)
@@ -82,6 +82,45 @@ def test_flash_decode_lengths(rkv, rko, ctx, D, L):
         assert np.abs(got[h] - want).max() <= 1e-5 * np.abs(want).max()
 
 
+@pytest.mark.parametrize("L", [200, 1000])
+def test_flash_decode_captured(rkv, rko, ctx, L):
+    """The drop-in in a HIP graph: each replay, with other rows and queries in
+    the same buffers, gives an eager call's bits."""
+    torch = _torch()
+    Hq, Hkv, D = 6, 2, 128
+    p = rkv.FlashDecodeParams(Hq, Hkv, L, 1024, D)
+    scratch, other = (torch.full((rkv.flash_decode_scratch_bytes(p),), 0xFF, dtype=torch.uint8, device="cuda")
+                      for _ in range(2))
+    out, want = torch.empty((Hq, D), device="cuda"), torch.empty((Hq, D), device="cuda")
+    k, v = (torch.empty(Hkv * L * rkv.row_bytes(D), dtype=torch.uint8, device="cuda") for _ in range(2))
+    q = torch.empty((Hq, D), device="cuda")
+
+    def fill(seed):
+        rng = np.random.default_rng(seed)
+        for t in (k, v):
+            t.copy_(torch.from_numpy(rko.q8_encode(rng.standard_normal(Hkv * L * D).astype(np.float32)).copy()
+                                     .view(np.uint8).reshape(-1)))
+        q.copy_(torch.from_numpy((rng.standard_normal((Hq, D)) / np.sqrt(D)).astype(np.float32)))
+        torch.cuda.synchronize()
+
+    fill(0)
+    side = torch.cuda.Stream()
+    rkv.flash_decode_q8(ctx, p, k, v, q, out, scratch, stream=side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        rkv.flash_decode_q8(ctx, p, k, v, q, out, scratch, stream=side)
+    for rep in range(4):
+        fill(rep + 1)
+        out.fill_(float("nan"))
+        rkv.flash_decode_q8(ctx, p, k, v, q, want, other)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want), rep
+    del graph
+
+
 @pytest.mark.parametrize("D,PT,Hkv,layers,first,count", [
     (128, 16, 4, 30, 7, 300),    # 3 tiles a workgroup, both edges part-filled
     (128, 64, 1, 1, 33, 62),     # odd rows: runs at odd multiples of 8 bytes
@@ -90,6 +129,8 @@ def test_flash_decode_lengths(rkv, rko, ctx, D, L):
     (256, 16, 3, 2, 5, 9),       # inside one tile
     (256, 128, 8, 2, 0, 1),
     (128, 32, 2, 2, 40, 0),      # no tokens: header and CRC of nothing
+    (256, 64, 2, 48, 3, 4100),   # 15 tiles a workgroup, both edges part-filled
+    (128, 16, 16, 56, 5, 1100),  # more streams than workgroups at once: 64 tiles each, the most
 ])
 def test_spill_edges(rkv, ctx, D, PT, Hkv, layers, first, count):
     torch = _torch()
