@@ -58,8 +58,7 @@ __device__ inline void load_src8(const void *src, uint64_t off, float v[8]) {
 // 8-row blocks share a tile).  65,619 rows of 16 sequences of odd lengths
 // (D 256, 2 kv heads, bf16): 59.5 us with neither, 54.8 with the chunks, 50.4
 // with both; 4101 rows of 8 sequences 9.65, 8.6, 8.3; 65,536 rows that start at
-// tiles 46.3 to 46.5 either way.  With another
-// form of the quads chunks of 1, 8 and 64 took 66.3, 63.0 and 66.0 us.
+// tiles 46.3 to 46.5 either way.
 template <int kAppRows>
 constexpr uint32_t kAppChunk = kAppRows == 32 ? 8 : 4;
 
@@ -247,10 +246,13 @@ __global__ __launch_bounds__(256) void append_kernel(AppendLaunch a) {
 
 // Export (gather) and import of positions [0, len) of one sequence: one
 // 128-thread workgroup per (tile of the positions, kv head), moving the tile
-// through an LDS image of its rows (rkv_rows.h).  HBM bound: a 32,768-token
-// sequence (D = 256, 2 kv heads, 35.7 MB each way and kind) took 77 us to
+// through an LDS image of its rows (rkv_rows.h).  A 32,768-token sequence (D =
+// 256, 2 kv heads, 17.8 MB read and 17.8 MB written per kind) took 77 us to
 // gather and 62 us to import with one thread per 34-byte block and byte
-// accesses; the tile form takes 15.9 and 13.2 us (4.5 and 5.4 TB/s).
+// accesses.  The tile form's gather takes 8.0 us for K and 17.0 for V, its
+// import 9.0 and 14.6 (kernel trace; 4.5, 2.1, 4.0 and 2.4 TB/s read and
+// written): K moves at about the rate of a large copy, V, whose lanes' 16
+// bytes lie 128 apart, at half of it.
 template <int D>
 __global__ __launch_bounds__(kRowsThreads) void gather_kernel(Geo g, const uint8_t *pages, const int32_t *bt,
                                                               int32_t len, int32_t kind, uint8_t *rows,

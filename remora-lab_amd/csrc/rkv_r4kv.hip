@@ -211,14 +211,16 @@ __global__ void spill_end_kernel(const uint32_t *crc_word, uint32_t finish, uint
   *reinterpret_cast<uint32_t *>(to) = *crc_word ^ finish;
 }
 
-// Spill: the body and its CRC32C in one launch.  Each
-// tile's rows leave for the body from the LDS image, and the CRC is taken
-// from the same image, so the body is not read back (the CRC as a second
-// pass over a 214 MB page took 115 us after a 128 us pack, and three one-word
-// launches about 4.7 us each; this launch takes 130 us, 3.3 TB/s
-// of its 428 MB of traffic, bound by the memory system: more or fewer
-// workgroups and deeper prefetch are slower).  Lane t holds words t, t + L, ... of the workgroup's
-// part of the body (L = TT*D/64, so a whole tile is 17 of them) and divides
+// Spill: the body and its CRC32C in one launch.  Each tile's rows leave for
+// the body from the LDS image, and the CRC is taken from the same image, so
+// the body is not read back (the CRC as a second pass over a 214 MB page took
+// 115 us after a 128 us pack; this launch takes 129, 3.3 TB/s of its 428 MB
+// of traffic).  HBM does not bound it: unpack_kernel moves the same bytes in 89.
+// The CRC is 10 us of the difference (118 against 128 us a spill without it);
+// the rest is the way these workgroups move tiles, of which two tiles ahead
+// (135 us), more workgroups (344 at a tile each) and fewer were slower.
+// Lane t holds words t, t + L, ... of the workgroup's part of the body
+// (L = TT*D/64, so a whole tile is 17 of them) and divides
 // them by P(x^(32 L)) as they come (crc_divide); a partly covered first tile
 // starts with zero words (which change nothing), and a partly covered last
 // one gets a workgroup of its own.  At the end the lanes' remainders are a
@@ -402,8 +404,9 @@ hipError_t launch_r4kv_pack(const R4kvLaunch &r, const uint8_t *pages, const int
   // a partly covered last tile behind others has a workgroup of its own
   const bool lone = m.n_tiles > 1 && (r.t0 + r.count) % TT != 0;
   m.n_main = m.n_tiles - (lone ? 1 : 0);
-  // one round of the seven workgroups that a CU's LDS holds, in even shares:
-  // each reduces its lanes' remainders and moves them to the body's end once
+  // one round of seven workgroups per CU, in even shares: each reduces its
+  // lanes' remainders and moves them to the body's end once.  Seven is what a
+  // CU's LDS holds at D = 256, where it was measured; at D = 128 12 would fit.
   const int64_t shares = std::clamp<int64_t>(7 * kComputeUnits / streams, 1, std::max(m.n_main, 1));
   m.per = (int32_t)std::clamp<int64_t>((m.n_main + shares - 1) / shares, 1, 64);  // a lane per tile's page
   const int32_t chunks = std::max<int32_t>(1, (m.n_main + m.per - 1) / m.per) + (lone ? 1 : 0);

@@ -10,8 +10,10 @@
 // LDS image of the run, 2 bytes at a time because blocks start on odd
 // halfwords.  K codes are rows already; V codes are dim-major, so a lane takes
 // 4 dims x 16 slots and transposes them 4x4 in registers (8 byte permutes per
-// 16 codes).  HBM bounds it: one workgroup of 128 threads per tile keeps
-// 8.5 KiB (D = 256) in flight, up to 16 of them per CU.
+// 16 codes).  One workgroup of 128 threads per tile keeps 8.5 KiB (D = 256) in
+// flight, up to 16 of them per CU.  K tiles move at about the rate of a large
+// copy, V tiles at half of it (rkv_append.hip has the times), likely because
+// the lanes' 16 bytes lie 128 apart and each access touches a line per lane.
 #pragma once
 
 #include "rkv_launch.h"

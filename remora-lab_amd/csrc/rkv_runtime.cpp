@@ -598,7 +598,9 @@ Plan plan_of(const rkv_kv_geometry *g, const rkv_decode_args *a, int32_t stages,
   // combine little.  Measured at 1, 2, 3, 4 and 8 tiles, us per call: 300
   // tokens (D 128) 12.4, 13.8, 13.8, 14.7, 19.1; 1024 tokens of 4 kv heads
   // 17.2, 19.6, 21.0, 22.6, 28.2; 32,768 tokens 22.1, 22.0, 20.7, 20.6, 24.4;
-  // four drafts (32 rows) on 4 x 1024 26.6, 24.0, 26.1, 21.8, 27.0.
+  // four drafts (32 rows) on 4 x 1024 26.6, 24.0, 26.1, 21.8, 27.0.  Between
+  // the few partitions of the first two and a full machine 2 stands for all:
+  // at 32,768 tokens 3 or 4 would be 1.3 us better.
   const int32_t tiles = (pl.max_len + pl.unit - 1) / pl.unit;
   pl.kmin = rows > 16 ? 4 : (B * tiles * g->kv_heads <= kFewPartitions ? 1 : 2);
   if (a->partition_tokens > 0) {
@@ -635,9 +637,10 @@ int32_t batch_rows_per_kv(const rkv_kv_geometry *g, const rkv_decode_args *a) {
 //            partition count of every entry (written by the decode)
 //   partials f32 (m, l) then o of every (kv head, partition, row)
 // Everything is written before it is read in the same call, so the
-// workspace needs no initialisation.  Every part grows with batch and
-// max_seq_len: a workspace sized for the largest call of a serving loop
-// holds every smaller one.
+// workspace needs no initialisation.  With device-chosen partitions no part
+// shrinks as batch or max_seq_len grows (up to 256 tokens there is none): a
+// workspace sized for the largest call of a serving loop holds every smaller
+// one.
 size_t align256(size_t n) { return (n + 255) / 256 * 256; }
 struct WsLayout {
   size_t hdr = 0, ml = 0, o = 0, total = 0;
@@ -648,13 +651,16 @@ WsLayout ws_layout(const rkv_kv_geometry *g, const rkv_decode_args *a, const Pla
   const size_t B = (size_t)std::max<int32_t>(a->batch, 0);
   const size_t out_rows = B * a->q_len * a->q_heads;
   const size_t prows = (size_t)g->kv_heads * pl.n_wg * batch_rows_per_kv(g, a);
-  // partitions of one entry: ceil(max_len / shortest partition), and with a
-  // device-chosen length no more than the target minus one per other entry
-  // (or the count at the longest length, where the search stops).  Shortest:
-  // what the device chooses when every entry is max_len long, up to the 8
-  // tiles below which only batches that do not fill the machine go (72
-  // sequences of about 2000 tokens, 9-tile partitions: 41.2 us with the one
-  // slice that this gives, 42.9 with two).
+  // An estimate of the partitions of one entry, for the slices below alone
+  // (memory and loops go by n_wg and by what the device writes): with a
+  // device-chosen length, what it chooses when every entry is max_len long, up
+  // to 8 tiles, and no more than the target minus one per other entry (or the
+  // count at the longest length, where the search stops).  One long entry
+  // among short ones can have more: 20 sequences, one of 4096 tokens and the
+  // others of 32, get one slice for 64 partitions and take 16.8 us a call
+  // (24.8 with partitions of 8 tiles).  72 sequences of about 2000 tokens,
+  // 9-tile partitions: 41.2 us with the one slice that this gives, 42.9 with
+  // two.
   const int64_t even = ((int64_t)B * ((pl.max_len + 31) / 32) + pl.target - 1) / pl.target;
   const int64_t shortest =
       pl.pt > 0 ? pl.pt : std::max<int64_t>(pl.kmin, std::min<int64_t>(even, 8)) * pl.unit;
